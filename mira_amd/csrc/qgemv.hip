@@ -392,6 +392,8 @@ __global__ void __launch_bounds__(256) w8gemv_kernel(const float* __restrict__ x
 
 // The weight-row stream for M <= 8, k_pad <= 4096: 16 columns per workgroup where
 // that gives every CU one, else 8 or 4 (n0 + COLS <= n_pad: n_pad % 32 == 0).
+constexpr int W8_MAX_STREAM_ROWS = 4;   // weight-only matmul rows above which the f32-MFMA tiles take over
+
 template <int PRE, int MR>
 static void ks_launch_m(const GemvArgs& g, const EpiDev& e, const RowIn& rin, hipStream_t stream) {
   const int64_t cus = device_cu_count();
@@ -556,8 +558,10 @@ extern "C" int mr_w8_matmul_f32(const float* x, int64_t ldx, const int8_t* b, co
   const int rc = mr::make_epi(epi, N, false, &e);
   if (rc != MR_OK) return rc;
   if (M == 0) return MR_OK;
-  // more than 16 rows: tiles on f32 MFMAs (the weights cross HBM once per 128 rows)
-  if (M > 16) {
+  // More rows: tiles on f32 MFMAs.  4096 x 4096 / 4096 x 1000 / 784 x 512, us: at 2 rows the stream
+  // takes 9.5 / 7.8 / 9.3 and the tiles 12.2 / 10.8 / 8.7, at 4 rows 13.7 / 9.1 / 12.9 and
+  // 11.4 / 10.7 / 7.8, at 8 rows 22.9 / 15.3 / 15.3 and 11.5 / 10.9 / 7.9.
+  if (M > mr::W8_MAX_STREAM_ROWS) {
     const int rt = mr::w8gemm_launch(x, ldx, b, w_scale, w_f16, k_pad, n_pad, M, N, K, e, static_cast<hipStream_t>(stream));
     if (rt != MR_EUNSUPPORTED) return rt;
   }

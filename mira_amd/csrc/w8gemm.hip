@@ -3,10 +3,12 @@
 // dequantize constant W[k][n] = fl32(q[k][n] * scale[n]) (mira/ops.py:581-589,
 // rounded on to f16 when the dequantize has dtype f16), then the epilogue
 // (mira/ops.py:217-219).  The weight-streaming kernel of qgemv.hip reads the
-// weights once per 8 rows; this one tiles the product on f32 MFMAs
-// (v_mfma_f32_32x32x2_f32), so the weights cross HBM once per 128 rows.
+// weights once per 8 rows; these tile the product on f32 MFMAs.  Batches with
+// fewer 128 x 128 tiles than CUs run on w8rows_f32_kernel (below), larger ones
+// and convolutions on w8gemm_f32_kernel (v_mfma_f32_32x32x2_f32), where the
+// weights cross HBM once per 128 rows.
 //
-// A workgroup owns a 128 x 128 tile and walks K in 64-element stages (one
+// w8gemm_f32_kernel: a workgroup owns a 128 x 128 tile and walks K in 64-element stages (one
 // 64-byte step of the packed weights).  Each stage's x slice (128 rows x 256
 // bytes of f32) and weight slice (128 rows x 64 int8) move global -> LDS by
 // buffer loads straight into LDS, double buffered; rows past M, columns past
@@ -228,6 +230,172 @@ __global__ void __launch_bounds__(256) w8gemm_f32_kernel(const W8GemmArgs g, con
     }
 }
 
+// Row blocks of a batch that leaves the 128 x 128 tiles short of CUs (17..~1000 rows at the usual
+// widths): a workgroup owns RB * 16 rows x CB * 16 columns and its 8 waves split K in steps of
+// 64, wave w taking steps w, w + 8, ...; the partial tiles meet in LDS at the end.  Split inside
+// the workgroup, K needs no workspace and no second launch, and RB follows the batch, so a
+// 33-row batch multiplies 48 rows instead of 128 and 4096 columns give 256 workgroups instead of
+// 32.  What bounds it is the f32 MFMA rate (v_mfma_f32_16x16x4_f32, 32 cycles) once a wave's
+// loads, one step ahead in registers, are covered: per step and lane one 16-byte run of a
+// column's weights, dequantized once and used by RB products, and one 64-byte run of each of its
+// RB rows (a row's step is 256 contiguous bytes over the 4 lane groups).  No LDS staging: no two
+// waves of a workgroup read the same bytes.
+// Measured (us per launch, 128 x 128 tiles -> this kernel): 4096 x 4096 at 17 / 33 / 100 / 300 / 700
+// rows 309 / 313 / 322 / 327 / 331 -> 17 / 25 / 53 / 146 / 288; 4096 x 1000 at 33 rows 312 -> 13;
+// 784 x 512 at 33 rows 73 -> 8; and against the 8-row weight stream, 4096 x 4096 at 4 / 8 / 16
+// rows 13.7 / 22.9 / 42.8 -> 11.4 / 12.4 / 13.2 (up to 4 rows stay there: qgemv.hip).
+template <int RB, int CB>
+__global__ void __launch_bounds__(512) w8rows_f32_kernel(const W8GemmArgs g, const EpiDev e) {
+  constexpr int WAVES = 8, LD = CB * 16 + 4;   // a row of partial sums, padded: 4 rows apart = 16 banks apart
+  __shared__ float part[WAVES][RB * 16][LD];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, kg = lane >> 4;
+  const int tile_n = blockIdx.x / g.tiles_m;
+  const int m0 = (blockIdx.x - tile_n * g.tiles_m) * RB * 16, n0 = tile_n * CB * 16;
+
+  const __amdgpu_buffer_rsrc_t rx =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g.x), 0, g.x_bytes, BUF_DWORD3);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(g.b), 0, g.b_bytes, BUF_DWORD3);
+
+  uint32_t x_off[RB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+    const int r = m0 + i * 16 + l16;
+    x_off[i] = r < g.M ? static_cast<uint32_t>((r * g.ldx + kg * 16) * 4) : W8_OOB;   // OOB + any step stays out of range
+  }
+  uint32_t b_off[CB];
+  float sc[CB];
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int n = n0 + j * 16 + l16;   // < n_pad: n_pad is a multiple of 32
+    b_off[j] = static_cast<uint32_t>(n * 64 + kg * 16);
+    sc[j] = g.ws[min(n, g.N - 1)];
+  }
+
+  // partial sums per K position modulo NA: short chains, so a decode-shaped batch (RB 1) rounds no
+  // more than the weight stream's 64 lanes do (4096 x 4096, error against 64 bits: the stream
+  // 1.59e-7, one chain per wave 4.1e-7, 4 chains 2.15e-7, 16 chains 1.26e-7; the 128 x 128 tiles 1.14e-6)
+  constexpr int NA = RB == 1 ? 16 : 1;
+  v4f acc[NA][RB][CB];
+#pragma unroll
+  for (int c = 0; c < NA; ++c)
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) acc[c][i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int KT = g.k_pad / W8K;
+  struct Step {
+    v4f x[RB][4];
+    v4i w[CB];
+  };
+  auto fetch = [&](Step& t, int kt) __attribute__((always_inline)) {
+    const uint32_t soff = static_cast<uint32_t>(kt) * static_cast<uint32_t>(g.n_pad) * 64u;
+#pragma unroll
+    for (int j = 0; j < CB; ++j) t.w[j] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[j] + soff, 0, 0);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        // K % 4 == 0 (checked on the host): 4 elements are all below K or all past it
+        const uint32_t off = kt * W8K + kg * 16 + q * 4 < g.K ? x_off[i] + static_cast<uint32_t>(kt * 256 + q * 16) : W8_OOB;
+        t.x[i][q] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
+      }
+  };
+  auto multiply = [&](const Step& t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        float w[CB];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          const int byte = __builtin_amdgcn_sbfe(t.w[j][q], kk * 8, 8);   // sign-extended int8
+          w[j] = __fmul_rn(static_cast<float>(byte), sc[j]);
+          if (g.w16) w[j] = round_f16(w[j]);
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+          for (int j = 0; j < CB; ++j)
+            acc[(q * 4 + kk) % NA][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(t.x[i][q][kk], w[j], acc[(q * 4 + kk) % NA][i][j], 0, 0, 0);
+      }
+  };
+
+  Step a, b;
+  int kt = wave;
+  if (kt < KT) fetch(a, kt);
+  for (; kt < KT; kt += 2 * WAVES) {
+    if (kt + WAVES < KT) fetch(b, kt + WAVES);
+    multiply(a);
+    if (kt + WAVES >= KT) break;
+    if (kt + 2 * WAVES < KT) fetch(a, kt + 2 * WAVES);
+    multiply(b);
+  }
+
+  // lane holds column l16 and rows 4 * kg .. + 3 of each block
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int h = NA / 2; h > 0; h >>= 1)
+#pragma unroll
+          for (int c = 0; c < h; ++c) acc[c][i][j][r] += acc[c + h][i][j][r];
+        part[wave][i * 16 + 4 * kg + r][j * 16 + l16] = acc[0][i][j][r];
+      }
+  __syncthreads();
+  for (int o = threadIdx.x; o < RB * 16 * CB * 16; o += 512) {
+    const int r = o / (CB * 16), c = o % (CB * 16);
+    const float y = ((part[0][r][c] + part[1][r][c]) + (part[2][r][c] + part[3][r][c])) +
+                    ((part[4][r][c] + part[5][r][c]) + (part[6][r][c] + part[7][r][c]));
+    const int row = m0 + r, col = n0 + c;
+    if (row < g.M && col < g.N) epi_store(e, epi_steps(e, y, row, col), row, col);
+  }
+}
+
+template <int RB, int CB>
+static void w8rows_start(const W8GemmArgs& g, const EpiDev& e, hipStream_t stream) {
+  W8GemmArgs a = g;
+  a.tiles_m = (g.M + RB * 16 - 1) / (RB * 16);
+  const unsigned grid = static_cast<unsigned>(a.tiles_m) * static_cast<unsigned>((g.N + CB * 16 - 1) / (CB * 16));
+  hipLaunchKernelGGL((w8rows_f32_kernel<RB, CB>), dim3(grid), dim3(512), 0, stream, a, e);
+}
+
+// Does this batch run on w8rows_f32_kernel?  Fewer 128 x 128 tiles than CUs leave CUs idle for a
+// whole tile's K loop (4096 x 4096: 192 tiles 331 -> 288 us here, 256 tiles 333 -> 375).
+static bool w8rows_pays(int64_t M, int64_t N) {
+  return ((M + W8T - 1) / W8T) * ((N + W8T - 1) / W8T) < device_cu_count();
+}
+
+// The widest blocks (fewest loads per product: 32 columns, up to 64 rows) that still give every CU
+// a workgroup; then the rows are spread evenly over the row blocks.
+static void w8rows_launch(const W8GemmArgs& g, const EpiDev& e, hipStream_t stream) {
+  const int64_t blocks = (int64_t(g.M) + 15) / 16, cus = device_cu_count();
+  auto grid = [&](int rb, int cb) { return ((blocks + rb - 1) / rb) * ((g.N + cb * 16 - 1) / (cb * 16)); };
+  int rb = static_cast<int>(blocks < 4 ? blocks : 4);
+  const int cb = grid(rb, 2) >= cus ? 2 : 1;
+  while (rb > 1 && grid(rb, cb) < cus) --rb;
+  const int64_t tiles_m = (blocks + rb - 1) / rb;
+  rb = static_cast<int>((blocks + tiles_m - 1) / tiles_m);
+  if (cb == 2) {
+    if (rb == 1) w8rows_start<1, 2>(g, e, stream);
+    else if (rb == 2) w8rows_start<2, 2>(g, e, stream);
+    else if (rb == 3) w8rows_start<3, 2>(g, e, stream);
+    else w8rows_start<4, 2>(g, e, stream);
+  } else {
+    if (rb == 1) w8rows_start<1, 1>(g, e, stream);
+    else if (rb == 2) w8rows_start<2, 1>(g, e, stream);
+    else if (rb == 3) w8rows_start<3, 1>(g, e, stream);
+    else w8rows_start<4, 1>(g, e, stream);
+  }
+}
+
 int w8gemm_launch(const float* x, int64_t ldx, const int8_t* b, const float* w_scale, int32_t w_f16, int64_t k_pad,
                   int64_t n_pad, int64_t M, int64_t N, int64_t K, const EpiDev& e, hipStream_t stream,
                   const mr_conv_geom* cg) {
@@ -252,6 +420,11 @@ int w8gemm_launch(const float* x, int64_t ldx, const int8_t* b, const float* w_s
     g.KH = cg->kh; g.KW = cg->kw; g.SH = cg->sh; g.SW = cg->sw; g.PH = cg->ph; g.PW = cg->pw; g.DH = cg->dh; g.DW = cg->dw;
   }
   g.b_bytes = static_cast<uint32_t>(k_pad * n_pad);
+  if (!cg && w8rows_pays(M, N)) {
+    w8rows_launch(g, e, stream);
+    MR_LAUNCH_CHECK("w8rows");
+    return MR_OK;
+  }
   const int64_t tiles = int64_t(g.tiles_m) * ((N + W8T - 1) / W8T);
   MR_REQUIRE(tiles < (int64_t(1) << 31), "w8gemm: too many tiles");
   if (cg)

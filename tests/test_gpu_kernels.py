@@ -355,7 +355,7 @@ def test_w8_matmul_bias_relu(lib, M, K, N, ldx):
 @pytest.mark.parametrize("M,K,N,ldx", [(17, 64, 33, 64), (128, 784, 512, 784), (300, 1024, 1000, 1028),
                                        (1000, 256, 130, 256), (40, 33, 20, 36)])
 def test_w8_matmul_tiled(lib, M, K, N, ldx):
-    """More than 16 rows: 128 x 128 f32-MFMA tiles (ragged M, N and K tails; the last case,
+    """More than 16 rows: f32-MFMA tiles (ragged M, N and K tails; the last case,
     K % 4 != 0, takes the 8-row weight stream instead)."""
     rng = np.random.default_rng(M * 7 + K + N)
     x = rng.standard_normal((M, ldx)).astype(np.float32)
@@ -370,6 +370,24 @@ def test_w8_matmul_tiled(lib, M, K, N, ldx):
     assert np.all(np.abs(y.astype(np.float64) - want) <= W8_TOL * bound)
     assert (y >= 0).all()
     assert bits_equal(yq, G.quantize_activation(y, 0.02).astype(np.int8))
+
+
+@pytest.mark.parametrize("M,K,N", [(5, 4096, 40), (16, 68, 16), (16, 512, 4096), (17, 448, 33), (33, 1000, 4100),
+                                   (48, 576, 8200), (49, 64, 1), (64, 520, 8192), (65, 1088, 4097), (700, 132, 4096),
+                                   (2100, 68, 2000)])
+def test_w8_matmul_row_tiles(lib, M, K, N):
+    """Every block shape of the row tiles (1..4 blocks of 16 rows by 16 or 32 columns) at its ragged
+    edges, K short of, at and past one step per wave, and (the last case: 272 tiles) the 128 x 128
+    tiles.  Bound: f32 sums of K products in any order stay within K * 2^-24 of sum |x||w|, and far
+    less in practice; 1e-5 holds for every K here, as for the shapes above."""
+    rng = np.random.default_rng(M * 3 + K + N)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    q = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    s = rng.uniform(0.001, 0.01, N).astype(np.float32)
+    deq = G.dequantize({"q": q, "scale": s, "axis": 1, "dtype": "f32"}).astype(np.float64)
+    y, yq = _run_w8(lib, x, K, q, s, [], next_xs=0.05)
+    assert np.all(np.abs(y - x.astype(np.float64) @ deq) <= W8_TOL * (np.abs(x).astype(np.float64) @ np.abs(deq)))
+    assert bits_equal(yq, G.quantize_activation(y, 0.05).astype(np.int8))
 
 
 def test_w8_matmul_tiled_f16_weights(lib):
