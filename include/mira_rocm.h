@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define MR_ABI_VERSION 12
+#define MR_ABI_VERSION 13
 
 enum mr_status {
   MR_OK = 0,
@@ -497,6 +497,74 @@ int mr_decode_commit(const float* logits, int64_t ldl, int32_t V, int32_t n_cach
                      int32_t* tokens, int64_t ld_tok, int32_t* t_io,
                      const int32_t* t_cur, int32_t prompt_len, int32_t T,
                      int64_t B, void* stream);
+
+/* ---- runs of row-local ops as one launch -------------------------------- */
+
+/* Ops whose result row r depends on row r of their inputs only. */
+enum mr_row_kind {
+  MR_ROW_QUANTIZE = 1,  /* mr_quantize_rows: x, ldx, d, yq, ldq, xs */
+  MR_ROW_LAYERNORM = 2, /* mr_layernorm_f32: x, ldx, d, gamma, beta, eps, round_f16,
+                           y, ldy, yq, ldq, xs; at most 512 elements per row */
+  MR_ROW_QMATMUL = 3,   /* mr_qmatmul: a, lda, b, k_pad, n_pad, d (= N), K, epi */
+  MR_ROW_ATTENTION = 4  /* mr_attention_decode_f32: x = q, ldx, the caches, the step's
+                           rows, mask, scale, heads, head_dim, keys (= T), y, ldy, yq,
+                           ldq, xs; heads * head_dim <= 256 */
+};
+
+/* The stage's f32 / int8 result is read by later stages of the run and by nothing
+ * else: it need not be stored (its buffer's contents are then undefined). */
+#define MR_ROW_ONLY_HERE_F32 1
+#define MR_ROW_ONLY_HERE_I8 2
+
+/* One op of a run, with the arguments of the entry point named above (the same
+ * requirements); fields the kind does not list are ignored. */
+typedef struct mr_row_stage {
+  int32_t kind;
+  int32_t round_f16;
+  int32_t d;
+  int32_t heads, head_dim, keys;
+  float eps, xs, scale;
+  int32_t flags;        /* MR_ROW_ONLY_HERE_* */
+  const float* x;
+  int64_t ldx;
+  const float* gamma;
+  const float* beta;
+  float* y;
+  int64_t ldy;
+  int8_t* yq;
+  int64_t ldq;
+  const int8_t* a;
+  int64_t lda;
+  const int8_t* b;
+  int64_t k_pad, n_pad, K;
+  const mr_epilogue* epi;
+  const float* k_cache;
+  const float* v_cache;
+  int64_t c_ld, c_bs;
+  const float* k_new;
+  int64_t ld_kn;
+  const float* v_new;
+  int64_t ld_vn;
+  const float* mask;
+} mr_row_stage;
+
+/* Bytes of the descriptors of a run of n stages (-1: not a run). */
+int64_t mr_row_chain_bytes(int32_t n);
+
+/* Check a run of n stages over `rows` rows and write its kernel descriptors
+ * (mr_row_chain_bytes(n) bytes of host memory, which the caller copies to the
+ * device and keeps) and its launch plan (4 values).  A stage may read what an
+ * earlier one of the run wrote, at the same row only, as whole rows or a slice
+ * of their columns.  Nothing is launched.  MR_EUNSUPPORTED when a stage is
+ * outside the limits above or the rows do not fit LDS: the caller then launches
+ * the ops one by one. */
+int mr_row_chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows,
+                         void* descriptors, int64_t bytes, int32_t* plan);
+
+/* Run a prepared run of stages over its rows in one launch.  Results are those of
+ * the entry points launched one after another, bit for bit. */
+int mr_row_chain(const void* descriptors, int64_t rows, const int32_t* plan,
+                 void* stream);
 
 #ifdef __cplusplus
 }

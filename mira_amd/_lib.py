@@ -10,7 +10,7 @@ from pathlib import Path
 from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "libmira_rocm.so"
-ABI_VERSION = 12
+ABI_VERSION = 13
 MAX_EPI = 8
 
 # enum mr_epi_fn
@@ -38,8 +38,13 @@ EXPORTS = [
     "mr_layernorm_f32", "mr_softmax_f32", "mr_bmm_f32", "mr_transpose_f32", "mr_copy_rows_f32",
     "mr_attention_decode_f32", "mr_decode_embed", "mr_decode_commit", "mr_elementwise_f32",
     "mr_elementwise_i32", "mr_cast_32", "mr_gather_rows_32", "mr_dynamic_slice_32", "mr_dynamic_update_slice_32",
-    "mr_argmax_f32", "mr_where_32",
+    "mr_argmax_f32", "mr_where_32", "mr_row_chain_bytes",
+    "mr_row_chain_prepare", "mr_row_chain",
 ]
+EUNSUPPORTED = 3
+# enum mr_row_kind
+ROW_QUANTIZE, ROW_LAYERNORM, ROW_QMATMUL, ROW_ATTENTION = 1, 2, 3, 4
+ROW_ONLY_HERE_F32, ROW_ONLY_HERE_I8 = 1, 2
 DT = {"f32": 0, "f16": 1, "i32": 2}       # enum mr_dtype
 DECODE_MAX_CACHES = 16      # MR_DECODE_MAX_CACHES
 
@@ -59,6 +64,18 @@ class Epilogue(C.Structure):
 class ConvGeom(C.Structure):
     _fields_ = [(n, C.c_int32) for n in
                 ("n", "h", "w", "c", "c_pad", "o", "oh", "ow", "kh", "kw", "sh", "sw", "ph", "pw", "dh", "dw")]
+
+
+class RowStage(C.Structure):
+    _fields_ = [*[(n, C.c_int32) for n in ("kind", "round_f16", "d", "heads", "head_dim", "keys")],
+                *[(n, C.c_float) for n in ("eps", "xs", "scale")], ("flags", C.c_int32),
+                ("x", C.c_void_p), ("ldx", C.c_int64), ("gamma", C.c_void_p), ("beta", C.c_void_p),
+                ("y", C.c_void_p), ("ldy", C.c_int64), ("yq", C.c_void_p), ("ldq", C.c_int64),
+                ("a", C.c_void_p), ("lda", C.c_int64), ("b", C.c_void_p),
+                *[(n, C.c_int64) for n in ("k_pad", "n_pad", "K")], ("epi", C.POINTER(Epilogue)),
+                ("k_cache", C.c_void_p), ("v_cache", C.c_void_p), ("c_ld", C.c_int64), ("c_bs", C.c_int64),
+                ("k_new", C.c_void_p), ("ld_kn", C.c_int64), ("v_new", C.c_void_p), ("ld_vn", C.c_int64),
+                ("mask", C.c_void_p)]
 
 
 class RocmError(RuntimeError):
@@ -116,6 +133,9 @@ _SIGS = {
     "mr_argmax_f32": ([_p, _i64, _i64, _p, _p], C.c_int),
     "mr_where_32": ([_p, _i32, C.POINTER(_i64), _p, C.POINTER(_i64), _p, C.POINTER(_i64), _p, C.POINTER(_i64), _p],
                     C.c_int),
+    "mr_row_chain_prepare": ([C.POINTER(RowStage), _i32, _i64, _p, _i64, C.POINTER(_i32)], C.c_int),
+    "mr_row_chain": ([_p, _i64, C.POINTER(_i32), _p], C.c_int),
+    "mr_row_chain_bytes": ([_i32], _i64),
     "mr_elementwise_f32": ([_i32, _p, C.POINTER(_i64), _p, C.POINTER(_i64), _p, C.POINTER(_i64), _i32, _p], C.c_int),
     "mr_decode_commit": ([_p, _i64, _i32, _i32, _p, _p, _p, _i64, _i64, _i32, _p, _i64, _p, _p, _i32, _i32, _i64, _p],
                          C.c_int),
@@ -145,7 +165,8 @@ def load(path: Optional[Path] = None) -> C.CDLL:
         fn.restype = res
     if lib.mr_abi_version() != ABI_VERSION:
         raise RocmError(f"{p}: ABI version {lib.mr_abi_version()} != {ABI_VERSION}")
-    for name, cls in (("mr_epi_step", EpiStep), ("mr_epilogue", Epilogue), ("mr_conv_geom", ConvGeom)):
+    for name, cls in (("mr_epi_step", EpiStep), ("mr_epilogue", Epilogue), ("mr_conv_geom", ConvGeom),
+                      ("mr_row_stage", RowStage)):
         if lib.mr_sizeof(name.encode()) != C.sizeof(cls):
             raise RocmError(f"{p}: sizeof({name}) {lib.mr_sizeof(name.encode())} != binding {C.sizeof(cls)}")
     _lib = lib

@@ -132,6 +132,7 @@ int64_t mr_sizeof(const char* name) {
   if (!std::strcmp(name, "mr_epi_step")) return sizeof(mr_epi_step);
   if (!std::strcmp(name, "mr_epilogue")) return sizeof(mr_epilogue);
   if (!std::strcmp(name, "mr_conv_geom")) return sizeof(mr_conv_geom);
+  if (!std::strcmp(name, "mr_row_stage")) return sizeof(mr_row_stage);
   return -1;
 }
 

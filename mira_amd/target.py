@@ -108,6 +108,12 @@ IMAGE_OPS = ("qconv2d", "conv2d", "maxpool2d", "pad", "reduce_mean")
 W8_STREAM_ROWS = 64   # mr_w8_matmul_f32 streams the weights once per 8 rows when K % 4 != 0
 F32IN_MAX_ROWS, F32IN_MAX_K = 8, 4096     # mr_qmatmul_f32in's decode shapes (k_pad <= 4096)
 LNIN_MAX_K = 1024                          # mr_qmatmul_lnin's rows (k_pad <= 1024)
+# Runs of row-local launches as one (_plan_row_chains): packed bytes of a q-op, and rows.  Four
+# K x K q-ops with two layernorms and residuals, us as launches / as a run (in a HIP graph):
+#   K = 64    1 row 17.9 / 14.3    512 rows 21.4 / 15.8    1024 rows 21.8 / 21.1
+#   K = 256   1 row 19.2 / 17.8    512 rows 27.4 / 20.6    1024 rows 28.0 / 27.1
+#   K = 384   1 row 19.5 / 26.2    512 rows 30.8 / 32.0    1024 rows 32.0 / 42.3
+ROW_CHAIN_WEIGHTS, ROW_CHAIN_ROWS = 64 << 10, 512
 
 
 _UNARY_CODES = {L.EPI_FN[f] for f in L.EPI_UNARY}
@@ -448,6 +454,8 @@ class RocmExecutable:
         self.acc: dict["Value", object] = {}      # debug int32 accumulators per q-op result
         self.kernel_counts: dict[str, int] = {}
         self.launch_cost: list[tuple[str, int, int]] = []
+        self.row_stages: list = []    # per launch: (rows, its mr_row_stage list), or None
+        self.col_operands: set = set()   # ids of epilogues with a computed operand that is not per row
         self.const_bytes = 0
         self._plan()
 
@@ -563,6 +571,87 @@ class RocmExecutable:
         for v in g.outputs:
             if v in self.consts and v not in self.dv:
                 self._const_dv(v)
+        self._plan_row_chains()
+
+    def _plan_row_chains(self) -> None:
+        """What launch() queues: `launches` in order, with each run of two or more neighbours
+        that are row-local over the same rows (row r of a result depends on row r of its inputs:
+        quantize, layernorm, qmatmul, decode attention) as one mr_row_chain launch.  A q-op
+        joins when its packed weights are at most ROW_CHAIN_WEIGHTS: every workgroup of the run
+        reads them through its own CU."""
+        self.program: list = []
+        run: list = []
+
+        def flush() -> None:
+            fn = self._row_chain(run) if len(run) > 1 else None
+            if fn is not None:
+                self.program.append(fn)
+            else:
+                self.program.extend(f for f, _ in run)
+            run.clear()
+
+        for (_name, fn), st in zip(self.launches, self.row_stages):
+            if st is None or st[0] > ROW_CHAIN_ROWS:
+                flush()
+                self.program.append(fn)
+                continue
+            if run and run[0][1][0] != st[0]:
+                flush()
+            run.append((fn, st))
+        flush()
+
+    def _row_chain(self, run: list):
+        """The launch of a run of row-local launches [(fn, (rows, stages))], or None when the
+        library declines it."""
+        torch = _t()
+        stages = [s for _, (_, ss) in run for s in ss]
+        n, rows = len(stages), run[0][1][0]
+        arr = (L.RowStage * n)(*stages)
+        if len(run) == len(self.launches):      # no other launch reads a result: only the outputs leave
+            out = [(t.data_ptr(), t.data_ptr() + t.nbytes()) for t in
+                   (self._src(v).f32.untyped_storage() for v in self.g.outputs)]
+            for s in arr:
+                y = s.epi.contents.out_f32 if s.kind == L.ROW_QMATMUL else s.y
+                s.flags = L.ROW_ONLY_HERE_I8
+                if y and not any(a <= y < b for a, b in out):
+                    s.flags |= L.ROW_ONLY_HERE_F32
+        size = self.lib.mr_row_chain_bytes(n)
+        host = np.zeros(size, np.uint8)
+        plan = (C.c_int32 * 4)()
+        rc = self.lib.mr_row_chain_prepare(arr, n, rows, host.ctypes.data, size, plan)
+        if rc == L.EUNSUPPORTED:
+            return None
+        L.check(rc, "mr_row_chain_prepare")
+        desc = torch.from_numpy(host).to(self.dev)
+        lib = self.lib
+        return lambda s: L.check(lib.mr_row_chain(desc.data_ptr(), rows, plan, s), "mr_row_chain")
+
+    def _quantize_stage(self, x, rows: int, cols: int, q, ld: int, xs: float) -> tuple:
+        return rows, [L.RowStage(kind=L.ROW_QUANTIZE, d=cols, x=x.data_ptr(), ldx=cols, yq=q.data_ptr(), ldq=ld, xs=xs)]
+
+    def _layernorm_stage(self, op: "Op", x, rows: int, d: int, gm, bt, y, yq, ld: int, xs: float) -> Optional[tuple]:
+        if any(v not in self.consts for v in op.inputs[1:3]):
+            return None
+        return rows, [L.RowStage(kind=L.ROW_LAYERNORM, round_f16=int(op.result.type.dtype == "f16"), d=d,
+                                 eps=float(op.attrs["eps"]), xs=xs, x=x.data_ptr(), ldx=d, gamma=gm.data_ptr(),
+                                 beta=bt.data_ptr(), y=_ptr(y), ldy=d, yq=_ptr(yq), ldq=ld)]
+
+    def _qmatmul_stage(self, xq, lda: int, b, kp: int, npad: int, M: int, N: int, K: int, e) -> Optional[tuple]:
+        if kp * npad > ROW_CHAIN_WEIGHTS or e.out_acc or id(e) in self.col_operands:
+            return None
+        return M, [L.RowStage(kind=L.ROW_QMATMUL, a=xq.data_ptr(), lda=lda, b=b.data_ptr(), k_pad=kp, n_pad=npad,
+                              d=N, K=K, epi=C.pointer(e))]
+
+    def _prologue_stage(self, first, M: int, K: int, b, kp: int, npad: int, N: int, e) -> Optional[tuple]:
+        """The stages of a q-op that makes its int8 rows itself: first(q, ld) gives the stage that
+        writes them, here to a buffer of the run's own."""
+        q = _t().empty((M, pack.row_stride_for(K)), dtype=_t().int8, device=self.dev)
+        a = first(q, q.stride(0))
+        m = self._qmatmul_stage(q, q.stride(0), b, kp, npad, M, N, K, e)
+        if a is None or m is None:
+            return None
+        self.keep.append(q)
+        return M, a[1] + m[1]
 
     def _padded_w8_input(self, op: "Op") -> bool:
         """A weight-only convolution over a graph input whose channel count is not a multiple
@@ -781,6 +870,12 @@ class RocmExecutable:
         return lambda s: L.check(lib.mr_qmatmul_lnin(x.data_ptr(), K, gm.data_ptr(), bt.data_ptr(), eps, f16, xs,
                                                      b.data_ptr(), kp, npad, M, N, K, C.byref(e), s),
                                  "mr_qmatmul_lnin")
+
+    def _lnin_stages(self, ln: "Op", xs: float, b, kp: int, npad: int, M: int, N: int, K: int, e) -> Optional[tuple]:
+        x = self._c_order(ln.inputs[0])
+        gm, bt = self._c_order(ln.inputs[1]), self._c_order(ln.inputs[2])
+        return self._prologue_stage(lambda q, ld: self._layernorm_stage(ln, x, M, K, gm, bt, None, q, ld, xs), M, K, b,
+                                    kp, npad, N, e)
 
     def _full_operand_reader(self, u: "Op", v: "Value") -> bool:
         """Does the q-op u read v only as its int8 input (inputs[0]: the copy v's producer
@@ -1069,7 +1164,8 @@ class RocmExecutable:
             for xs, (q, ld) in d.i8.items():
                 self._add("input", lambda s, q=q, ld=ld, xs=xs: L.check(
                     lib.mr_quantize_rows(stage.data_ptr(), rows, cols, cols, q.data_ptr(), ld, xs, s),
-                    "mr_quantize_rows"), nbytes=4 * rows * cols + rows * ld)
+                    "mr_quantize_rows"), nbytes=4 * rows * cols + rows * ld,
+                    stages=self._quantize_stage(stage, rows, cols, q, ld, xs))
 
     def _upload(self, arr: np.ndarray, dtype=None):
         torch = _t()
@@ -1111,11 +1207,14 @@ class RocmExecutable:
             return self._const_dv(v)
         return self.dv[v]
 
-    def _add(self, name: str, fn: Callable[[int], None], nbytes: int = 0, nops: int = 0) -> None:
+    def _add(self, name: str, fn: Callable[[int], None], nbytes: int = 0, nops: int = 0,
+             stages: Optional[tuple] = None) -> None:
         """Append a launch; nbytes/nops are its algorithmic HBM bytes and integer ops (each
-        operand read once, each result written once; 2 ops per multiply-accumulate)."""
+        operand read once, each result written once; 2 ops per multiply-accumulate); `stages`,
+        of a row-local launch, its rows and the stages it is as part of a run."""
         self.launches.append((name, fn))
         self.launch_cost.append((name, int(nbytes), int(nops)))
+        self.row_stages.append(stages)
         self.kernel_counts[name] = self.kernel_counts.get(name, 0) + 1
 
     @staticmethod
@@ -1145,7 +1244,7 @@ class RocmExecutable:
         lib, src, rows, cols = self.lib, d.f32, d.rows, d.cols
         self._add("quantize", lambda s: L.check(lib.mr_quantize_rows(src.data_ptr(), rows, cols, cols, q.data_ptr(),
                                                                      ld, xs, s), "mr_quantize_rows"),
-                  nbytes=4 * rows * cols + rows * ld)
+                  nbytes=4 * rows * cols + rows * ld, stages=self._quantize_stage(src, rows, cols, q, ld, xs))
         return q, ld
 
     def _finish_i8(self, d: DevValue, fused: Optional[float]) -> None:
@@ -1178,6 +1277,8 @@ class RocmExecutable:
                 mode, t, ld = self._const_operand(v, rshape, is_conv)
             else:
                 mode = _bcast_mode(v.type.shape, rshape, is_conv)
+                if mode not in (L.BC_FULL, L.BC_ROW):
+                    self.col_operands.add(id(e))
                 t = self.dv[v].f32
                 ld = out.cols if mode == L.BC_FULL else 1
                 if self.dv[v].half:
@@ -1255,11 +1356,13 @@ class RocmExecutable:
         lib, kp, npad = self.lib, bl.shape[1], bl.shape[0]
         if ln is not None:
             self._add("qmatmul", self._lnin_launch(ln, xs, b, kp, npad, M, N, K, e),
-                      nbytes=4 * M * K + 8 * K + K * N + 8 * N + 4 * M * N, nops=2 * M * N * K)
+                      nbytes=4 * M * K + 8 * K + K * N + 8 * N + 4 * M * N, nops=2 * M * N * K,
+                      stages=self._lnin_stages(ln, xs, b, kp, npad, M, N, K, e))
         else:
             self._add("qmatmul", lambda s: L.check(
                 lib.mr_qmatmul(xq.data_ptr(), lda, b.data_ptr(), kp, npad, M, N, K, C.byref(e), s), "mr_qmatmul"),
-                nbytes=M * K + K * N + 8 * N + 4 * M * N, nops=2 * M * N * K)
+                nbytes=M * K + K * N + 8 * N + 4 * M * N, nops=2 * M * N * K,
+                stages=self._qmatmul_stage(xq, lda, b, kp, npad, M, N, K, e))
 
     def _emit_qmatmul(self, op: "Op") -> None:
         if op in self.row_group:
@@ -1286,11 +1389,13 @@ class RocmExecutable:
         lib, kp, npad = self.lib, bl.shape[1], bl.shape[0]
         if ln is not None:
             self._add("qmatmul", self._lnin_launch(ln, xs, b, kp, npad, M, N, K, e),
-                      nbytes=4 * M * K + 8 * K + K * N + self._epi_bytes(e, M, N), nops=2 * M * N * K)
+                      nbytes=4 * M * K + 8 * K + K * N + self._epi_bytes(e, M, N), nops=2 * M * N * K,
+                      stages=self._lnin_stages(ln, xs, b, kp, npad, M, N, K, e))
         else:
             self._add("qmatmul", lambda s: L.check(
                 lib.mr_qmatmul(xq.data_ptr(), lda, b.data_ptr(), kp, npad, M, N, K, C.byref(e), s), "mr_qmatmul"),
-                nbytes=M * K + K * N + self._epi_bytes(e, M, N), nops=2 * M * N * K)
+                nbytes=M * K + K * N + self._epi_bytes(e, M, N), nops=2 * M * N * K,
+                stages=self._qmatmul_stage(xq, lda, b, kp, npad, M, N, K, e))
         self._finish_i8(out, fused)
 
     def _emit_qmatmul_f32in(self, op: "Op", x) -> None:
@@ -1311,7 +1416,9 @@ class RocmExecutable:
         lib, kp, npad = self.lib, bl.shape[1], bl.shape[0]
         self._add("qmatmul", lambda s: L.check(
             lib.mr_qmatmul_f32in(x.data_ptr(), K, xs, b.data_ptr(), kp, npad, M, N, K, C.byref(e), s),
-            "mr_qmatmul_f32in"), nbytes=4 * M * K + K * N + self._epi_bytes(e, M, N), nops=2 * M * N * K)
+            "mr_qmatmul_f32in"), nbytes=4 * M * K + K * N + self._epi_bytes(e, M, N), nops=2 * M * N * K,
+            stages=self._prologue_stage(lambda q8, ld: self._quantize_stage(x, M, K, q8, ld, xs), M, K, b, kp, npad, N,
+                                        e))
         self._finish_i8(out, fused)
 
     def _emit_matmul(self, op: "Op") -> None:
@@ -1360,7 +1467,13 @@ class RocmExecutable:
             args[7], args[8].data_ptr(), args[9], args[10].data_ptr(), scale, Bn, H, hd, T, y.data_ptr(), D,
             _ptr(q8), ld8, xs, s), "mr_attention_decode_f32"),
             nbytes=4 * (2 * Bn * (T + 1) * D + Bn * D + (T + 1)) + 4 * Bn * D + (Bn * ld8 if q8 is not None else 0),
-            nops=4 * Bn * (T + 1) * D)
+            nops=4 * Bn * (T + 1) * D,
+            stages=(Bn, [L.RowStage(kind=L.ROW_ATTENTION, heads=H, head_dim=hd, keys=T, xs=xs, scale=scale,
+                                    x=q.data_ptr(), ldx=q.stride(0), y=y.data_ptr(), ldy=D, yq=_ptr(q8), ldq=ld8,
+                                    k_cache=kc.data_ptr(), v_cache=vc.data_ptr(), c_ld=c_ld, c_bs=c_bs,
+                                    k_new=kn.data_ptr(), ld_kn=kn.stride(0), v_new=vn.data_ptr(),
+                                    ld_vn=vn.stride(0), mask=mask.data_ptr())])
+            if a["mask"] in self.g.inputs or a["mask"] in self.consts else None)
         self._finish_i8(out, None)
 
     def _emit_w8_matmul(self, op: "Op") -> None:
@@ -1797,7 +1910,8 @@ class RocmExecutable:
         self._add("layernorm", lambda s: L.check(lib.mr_layernorm_f32(
             x.data_ptr(), rows, d, gm.data_ptr(), bt.data_ptr(), eps, f16, _ptr(y), _ptr(yq), ld, xs, s),
             "mr_layernorm_f32"),
-            nbytes=4 * rows * d + 8 * d + (4 * rows * d if y is not None else 0) + rows * ld)
+            nbytes=4 * rows * d + 8 * d + (4 * rows * d if y is not None else 0) + rows * ld,
+            stages=self._layernorm_stage(op, x, rows, d, gm, bt, y, yq, ld, xs))
         if out.nhwc:
             self._publish(out, y)
         else:
@@ -2239,7 +2353,7 @@ class RocmExecutable:
         """Queue every kernel of the segment on the current stream, starting from the f32 inputs
         already on the device (quantizing them is part of the work)."""
         stream = _t().cuda.current_stream(self.dev).cuda_stream
-        for _name, fn in self.launches:
+        for fn in self.program:
             fn(stream)
 
     def download(self) -> dict:
