@@ -362,7 +362,7 @@ static int expand_dw_run(const char* fn, const int8_t* x, int64_t ldx, const int
                  (!dw.out_f32 || (dw.ldo % 4 == 0 && aligned16(dw.out_f32))) && aligned16(dw.col_ptr),
              "%s: depthwise outputs and bias must be aligned for 4-channel runs", fn);
   if (G.n == 0) return MR_OK;
-  const int T = G.sh == 1 && oh >= 14 ? 14 : 7;
+  int T = G.sh == 1 && oh >= 14 ? 14 : 7;
   ExpandDwArgs a = {};
   a.x = x;
   a.b = b;
@@ -373,9 +373,16 @@ static int expand_dw_run(const char* fn, const int8_t* x, int64_t ldx, const int
   if (stem) {
     a.Hin = stem->h; a.Win = stem->w; a.SS = stem->sh;
   }
+  const int n_cb = (G.c + 31) / 32;
+  auto workgroups = [&](int t) { return int64_t(G.n) * ((ow + t - 1) / t) * ((oh + t - 1) / t) * n_cb; };
+  // A grid that leaves CUs idle is as slow as one tile: smaller tiles spread it, at the price of more
+  // halo (14: 1.31 expanded pixels per output, 7: 1.65; stride 2, 7: 1.15 per input, 4: 1.27).
+  // MobileNetV2 at batch 1 / 4 / 8, us: stride 1, 112 x 112 x 32 (64 / 256 / 512 workgroups) 8.9 / 9.3 /
+  // 10.4 -> 5.4 / 7.4 / 11.9; 56 x 56 x 144 (80 / 320 / 640) 8.8 / 9.6 / 11.5 -> 5.8 / 7.9 / 14.9;
+  // stride 2 to 28 x 28 x 144 (80 / 320 / 640) 6.3 / 7.0 / 8.1 -> 4.7 / 5.9 / 8.9.
+  if (workgroups(T) <= device_cu_count() * 5 / 4 && (T == 14 || (G.sh == 2 && !stem))) T = T == 14 ? 7 : 4;
   a.tiles_w = (ow + T - 1) / T;
   a.tiles = a.tiles_w * ((oh + T - 1) / T);
-  const int n_cb = (G.c + 31) / 32;
   const int64_t total = int64_t(G.n) * a.tiles;
   MR_REQUIRE(total < (int64_t(1) << 31), "%s: too many tiles", fn);
   a.total = static_cast<int32_t>(total);
@@ -389,7 +396,8 @@ static int expand_dw_run(const char* fn, const int8_t* x, int64_t ldx, const int
     else if (T == 14) expand_dw_launch<1, 14, 64, true>(a, ex, dw, grid, s);
     else expand_dw_launch<1, 7, 64, true>(a, ex, dw, grid, s);
   } else {
-    if (G.sh == 2) expand_dw_kp<2, 7>(k_pad, a, ex, dw, grid, s);
+    if (T == 4) expand_dw_kp<2, 4>(k_pad, a, ex, dw, grid, s);
+    else if (G.sh == 2) expand_dw_kp<2, 7>(k_pad, a, ex, dw, grid, s);
     else if (T == 14) expand_dw_kp<1, 14>(k_pad, a, ex, dw, grid, s);
     else expand_dw_kp<1, 7>(k_pad, a, ex, dw, grid, s);
   }
