@@ -23,7 +23,7 @@ LIB = PKG / "libmira_rocm.so"
 ARCH = "gfx950"
 
 SOURCES = ["abi.hip", "quantize.hip", "qgemm.hip", "qgemv.hip", "w8gemm.hip", "misc.hip", "stem.hip", "decode.hip", "expand_dw.hip", "loop.hip",
-           "rowchain.hip"]
+           "rowchain.hip", "qrows.hip"]
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",

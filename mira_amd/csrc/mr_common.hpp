@@ -310,6 +310,11 @@ int make_epi(const mr_epilogue* epi, int64_t cols, bool need_scale, EpiDev* out,
 int gemv_launch(const int8_t* a, int64_t lda, const int8_t* b, int64_t k_pad, int64_t n_pad, int64_t M, int64_t N,
                 const EpiDev& e, hipStream_t stream);
 
+// int8 matmul (cg NULL: rows of lda bytes) or convolution of a small result, K split over a
+// workgroup's waves (qrows.hip); MR_EUNSUPPORTED where the tiles of qgemm.hip are the better ones.
+int qrows_launch(const int8_t* x, int64_t lda, const mr_conv_geom* cg, const int8_t* b, int64_t k_pad, int64_t n_pad,
+                 int64_t M, int64_t N, const EpiDev& e, hipStream_t stream);
+
 // Weight-only int8 matmul of many rows on f32 MFMAs (w8gemm.hip); MR_EUNSUPPORTED when K
 // or ldx is not a multiple of 4 or an operand reaches 2 GiB.
 // With a conv geometry, the implicit-GEMM convolution of an NHWC f32 image (C % 4 == 0).

@@ -965,6 +965,8 @@ int mr_qmatmul(const int8_t* a, int64_t lda, const int8_t* b, int64_t k_pad, int
              "mr_qmatmul: operands of 2 GiB or more are not supported (32-bit buffer offsets)");
   g.a_bytes = static_cast<uint32_t>(M * lda);
   g.b_bytes = static_cast<uint32_t>(k_pad * n_pad);
+  rc = mr::qrows_launch(a, lda, nullptr, b, k_pad, n_pad, M, N, e, static_cast<hipStream_t>(stream));
+  if (rc != MR_EUNSUPPORTED) return rc;
   return mr::launch<mr::A_DENSE>(g, e, static_cast<hipStream_t>(stream));
 }
 
@@ -1004,10 +1006,12 @@ int mr_qconv2d(const int8_t* x, const mr_conv_geom* cg, const int8_t* b, int64_t
              "overflow", (long long)mr::MAX_EXACT_K);
   MR_REQUIRE(mr::aligned16(x) && mr::aligned16(b), "mr_qconv2d: operands must be 16-byte aligned");
   mr::EpiDev e;
-  const int rc = mr::make_epi(epi, G.o, true, &e, true);
+  int rc = mr::make_epi(epi, G.o, true, &e, true);
   if (rc != MR_OK) return rc;
   const int64_t M = int64_t(G.n) * oh * ow;
   if (M == 0) return MR_OK;
+  rc = mr::qrows_launch(x, 0, cg, b, k_pad, n_pad, M, G.o, e, static_cast<hipStream_t>(stream));
+  if (rc != MR_EUNSUPPORTED) return rc;
   e.nt_f32 = mr::stream_f32(e, M);
   mr::GemmArgs g = {};
   g.a = x;

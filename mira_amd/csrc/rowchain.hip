@@ -23,10 +23,10 @@
 //    are loaded before the barrier in front of it.
 //
 // Measured, against the launches: the 16 of a two-layer D = 64 decode step over 272 keys for 512
-// sequences 140.4 -> 59.9 us, one sequence's greedy decode of it 69.0 -> 44.0 us a token (40 of
-// them here: 1.2-2 us a stage, 5.5 us an attention), the three of one attention half
-// (layernorm, projections, attention; 512 sequences, 71 MB of cache, 14 us at 5.2 TB/s) 23.7 -> 20.1, a quantize and a 256 x 64 x 10 dense layer
-// 10.8 -> 5.7.
+// sequences 140.4 -> 59.9 us; one sequence's greedy decode of it 69.0 -> 44.0 us a token, about 36
+// of them here (1.2-2 us a stage, 5.5 us an attention); one attention half (layernorm,
+// projections, attention) of 512 sequences, 71 MB of cache, 23.7 -> 20.1; a quantize and a
+// 256 x 64 x 10 dense layer 10.8 -> 5.7.
 #include "mr_common.hpp"
 #include "np_sum.hpp"
 
