@@ -159,6 +159,13 @@ int mr_quantize_nchw_nhwc(const float* x, int32_t n, int32_t c, int32_t h, int32
 int mr_quantize_f16_nchw_nhwc(const float* x, int32_t n, int32_t c, int32_t h, int32_t w,
                               int8_t* q, int32_t c_pad, float xs, void* stream);
 
+/* Both copies of an image that enters a segment, in one pass over it: the NHWC
+ * f32 copy y[n][h][w][c] (of f32(f16(x)) when round_f16) and, if q, the int8 copy of
+ * those values as mr_quantize_nchw_nhwc writes it.  n < 65536. */
+int mr_image_in_f32(const float* x, int32_t n, int32_t c, int32_t h, int32_t w,
+                    int32_t round_f16, float* y, int8_t* q, int32_t c_pad, float xs,
+                    void* stream);
+
 /* ---- K2/K3: int8 GEMM with fused dequant/epilogue/requant -------------- */
 
 /* Replaces mira/ops.py:616-620 _qmatmul_ref (after quantize_activation):

@@ -1141,19 +1141,21 @@ class RocmExecutable:
         self.staging[v] = stage
         d = self._new_dv(v, with_i8=True)
         cast16 = any(op.inputs[0] is v for op in self.input_casts)
-        # an image that only feeds q-ops is quantized straight from its f16 rounding
-        fused16 = cast16 and d.nhwc and d.f32 is None
-        if cast16 and not fused16:
+        # an image's copies are made straight from its f16 rounding
+        if cast16 and not d.nhwc:
             self._round_f16(stage, stage)
-        quant_nchw = lib.mr_quantize_f16_nchw_nhwc if fused16 else lib.mr_quantize_nchw_nhwc
+        quant_nchw = lib.mr_quantize_f16_nchw_nhwc if cast16 else lib.mr_quantize_nchw_nhwc
         if d.nhwc:
             n, c, h, w = v.type.shape
-            if d.f32 is not None:
+            i8 = dict(d.i8)
+            if d.f32 is not None:       # with the first int8 copy, in one pass over the image
                 dst = d.f32
-                self._add("input", lambda s: L.check(lib.mr_nchw_to_nhwc_f32(stage.data_ptr(), n, c, h, w,
-                                                                             dst.data_ptr(), s), "mr_nchw_to_nhwc_f32"),
-                          nbytes=8 * n * c * h * w)
-            for xs, (q, cp) in d.i8.items():
+                xs0 = next(iter(i8), None)
+                q0, cp0 = i8.pop(xs0, (None, 0))
+                self._add("input", lambda s: L.check(lib.mr_image_in_f32(
+                    stage.data_ptr(), n, c, h, w, int(cast16), dst.data_ptr(), _ptr(q0), cp0, xs0 or 1.0, s),
+                    "mr_image_in_f32"), nbytes=8 * n * c * h * w + n * h * w * cp0)
+            for xs, (q, cp) in i8.items():
                 self._add("input", lambda s, q=q, cp=cp, xs=xs: L.check(
                     quant_nchw(stage.data_ptr(), n, c, h, w, q.data_ptr(), cp, xs, s),
                     "mr_quantize_nchw_nhwc"), nbytes=4 * n * c * h * w + n * h * w * cp)
