@@ -560,7 +560,7 @@ int64_t mr_row_chain_bytes(int32_t n);
 
 /* Check a run of n stages over `rows` rows and write its kernel descriptors
  * (mr_row_chain_bytes(n) bytes of host memory, which the caller copies to the
- * device and keeps) and its launch plan (4 values).  A stage may read what an
+ * device and keeps) and its launch plan (5 values).  A stage may read what an
  * earlier one of the run wrote, at the same row only, as whole rows or a slice
  * of their columns.  Nothing is launched.  MR_EUNSUPPORTED when a stage is
  * outside the limits above or the rows do not fit LDS: the caller then launches

@@ -7,7 +7,7 @@
 //
 // What bounds it: at decode shapes a launch of a few rows takes 4-11 us, nearly all of it
 // launch, drain and first-touch latency (a 512-row x 64 x 64 projection took 9.9 us).  Here an
-// op is a barrier and its own instructions: 16 waves share 4 SIMDs, so an instruction that all
+// op is a barrier and its own instructions: 16 waves (W) share 4 SIMDs, so an instruction that all
 // of them run costs 16 clocks, and a stage's time is its instruction count as much as its
 // loads.  The price is that each workgroup reads every weight byte of the run through its own
 // CU, so the caller keeps runs to weights that are small next to a launch
@@ -23,9 +23,9 @@
 //    are loaded before the barrier in front of it.
 //
 // Measured, against the launches: the 16 of a two-layer D = 64 decode step over 272 keys for 512
-// sequences 140.4 -> 59.9 us; one sequence's greedy decode of it 69.0 -> 44.0 us a token, about 36
+// sequences 140.4 -> 56.8 us; one sequence's greedy decode of it 69.0 -> 44.0 us a token, about 36
 // of them here (1.2-2 us a stage, 5.5 us an attention); one attention half (layernorm,
-// projections, attention) of 512 sequences, 71 MB of cache, 23.7 -> 20.1; a quantize and a
+// projections, attention) of 512 sequences, 71 MB of cache, 23.7 -> 19.4; a quantize and a
 // 256 x 64 x 10 dense layer 10.8 -> 5.7.
 #include "mr_common.hpp"
 #include "np_sum.hpp"
@@ -84,7 +84,6 @@ typedef const __attribute__((address_space(4))) RowStage* RowStageP;
 
 enum { ROW_LOAD = 0, ROW_F16 = 1, ROW_NO_BARRIER = 2 };   // a kind of the library's own; flags
 
-constexpr int ROW_WAVES = 16;
 constexpr int ROW_BATCH = 5;     // attention: key rows a lane has in flight (5 x 16 bytes of K and of V)
 constexpr int ROW_AHEAD = 2;     // qmatmul: epilogue steps whose column operands are loaded ahead
 
@@ -153,6 +152,7 @@ __device__ __forceinline__ v4i row_weights(const RowStage& st, int n, int kg, in
   return *reinterpret_cast<const MR_GLOBAL v4i*>(in_memory(st.b) + off);
 }
 
+template <int W>
 __device__ __forceinline__ void look_ahead(const RowStage& st, const RowGroup& g, Ahead& a) {
   if (st.kind == MR_ROW_QMATMUL) {
     if (g.wave * 16 >= st.d) return;
@@ -177,21 +177,23 @@ __device__ __forceinline__ void look_ahead(const RowStage& st, const RowGroup& g
 }
 
 // the workgroup's rows of a value made outside the run, d words each
+template <int W>
 __device__ __forceinline__ void row_load(const RowStage& st, const RowGroup& g) {
   for (int r = 0; r < g.nr; ++r) {
     const MR_GLOBAL int* src = reinterpret_cast<const MR_GLOBAL int*>(reinterpret_cast<uint64_t>(st.x) + (g.r0 + r) * st.ld_x);
     MR_LDS int* dst = g.at<int>(st.y_at + r * st.ldy);
-    for (int c = g.wave * 64 + g.lane; c < st.d; c += ROW_WAVES * 64) dst[c] = src[c];
+    for (int c = g.wave * 64 + g.lane; c < st.d; c += W * 64) dst[c] = src[c];
   }
 }
 
 // clip(rint(x / xs)) of the workgroup's rows, the bytes up to the row stride zeroed
+template <int W>
 __device__ __forceinline__ void row_quantize(const RowStage& st, const RowGroup& g) {
   const RowOut out(st, g);
   for (int r = 0; r < g.nr; ++r) {
     const MR_GLOBAL float* src =
         reinterpret_cast<const MR_GLOBAL float*>(reinterpret_cast<uint64_t>(st.x) + (g.r0 + r) * st.ld_x);
-    for (int c = g.wave * 64 + g.lane; c < st.ldq; c += ROW_WAVES * 64) {
+    for (int c = g.wave * 64 + g.lane; c < st.ldq; c += W * 64) {
       int8_t v = 0;
       if (c < st.d) v = quantize_one(st.x_at >= 0 ? g.at<float>(st.x_at)[r * st.ldx + c] : src[c], st.xs);
       out.put8(r, c, v);
@@ -199,7 +201,7 @@ __device__ __forceinline__ void row_quantize(const RowStage& st, const RowGroup&
   }
 }
 
-// one wave per row (at most ROW_MAX_ROWS = ROW_WAVES of them), as layernorm_kernel
+// one wave per row (at most as many rows as waves), as layernorm_kernel
 __device__ __forceinline__ void row_layernorm(const RowStage& st, const RowGroup& g, const Ahead& ahead) {
   const int r = g.wave, d = st.d;
   if (r >= g.nr) return;
@@ -233,13 +235,14 @@ __device__ __forceinline__ void row_layernorm(const RowStage& st, const RowGroup
 // 16 kg .. +15 of each 64-byte step, of input row l16 (any row past the workgroup's) and of
 // weight row n0 + l16 (1 KB contiguous per wave and step); its results are column l16, rows
 // 4 kg .. +3.  Bytes past the end of an input row meet zero weights.
+template <int W>
 __device__ __forceinline__ void row_qmatmul(const RowStage& st, const RowGroup& g, Ahead& ahead) {
   const int N = st.d, KT = st.k_tiles;
   if (g.wave * 16 >= N) return;
   const RowOut out(st, g);
   const int l16 = g.lane & 15, kg = g.lane >> 4;
   const MR_LDS int8_t* a = g.at<int8_t>(st.a_at) + min(l16, g.nr - 1) * st.lda + kg * 16;
-  for (int n0 = g.wave * 16; n0 < N; n0 += ROW_WAVES * 16) {
+  for (int n0 = g.wave * 16; n0 < N; n0 += W * 16) {
     const int col = min(n0 + l16, N - 1);
     if (n0 != g.wave * 16) {                  // past what look_ahead loaded
       ahead.scale = in_memory(st.col_scale)[col];
@@ -290,7 +293,7 @@ __device__ __forceinline__ void row_qmatmul(const RowStage& st, const RowGroup& 
   }
 }
 
-// Decode attention of the workgroup's sequences, ROW_WAVES / rpw waves each, bit for bit
+// Decode attention of the workgroup's sequences, W / rpw waves each, bit for bit
 // attention_decode_kernel's arithmetic: a score is one chain of multiply-adds over the head's
 // columns, value rows l, l + 64, ... are one chain per l, and the 64 chains meet in a butterfly
 // from 32 down (an int8 step behind it may flip with any other order, and with it a greedy
@@ -300,15 +303,15 @@ __device__ __forceinline__ void row_qmatmul(const RowStage& st, const RowGroup& 
 // wave's loads are whole rows, the butterfly's first steps stay in the wave (slots), the next
 // in registers (passes), and the rest meet in LDS (waves).  Scores pass along the HD / 4 lanes
 // of a head, each adding its 4 columns.
-//   work: [rpw][H][T + 1] scores, then [ROW_WAVES][64] float4 partial sums
-template <int HD>
+//   work: [rpw][H][T + 1] scores, then [W][64] float4 partial sums
+template <int W, int HD>
 __device__ __forceinline__ void row_attention(const RowStage& st, const RowGroup& g, MR_LDS float* work) {
   const RowOut out(st, g);
   constexpr int HL = HD / 4;                       // lanes that share a head's part of a row
   const int H = st.H, T = st.T, D = H * HD, L = D / 4, nj = T + 1, lane = g.lane;
   const int lp_log2 = L <= 1 ? 0 : 32 - __builtin_clz(L - 1), LP = 1 << lp_log2;
   const int slot = lane >> lp_log2, c = lane & (LP - 1), h = c / HL;
-  const int wps = ROW_WAVES / g.rpw;               // waves per sequence
+  const int wps = W / g.rpw;               // waves per sequence
   const int s = g.wave / wps, ws = g.wave - s * wps;
   const int passes = LP > wps ? LP / wps : 1;
   const bool on = c < L && s < g.nr && ws < LP;
@@ -365,7 +368,7 @@ __device__ __forceinline__ void row_attention(const RowStage& st, const RowGroup
     }
   }
   lds_store_barrier();
-  for (int job = g.wave; job < g.nr * H; job += ROW_WAVES) {
+  for (int job = g.wave; job < g.nr * H; job += W) {
     MR_LDS float* row = work + job * nj;
     float m = -__builtin_inff(), sum = 0.0f, e[ROW_BATCH];
 #pragma unroll
@@ -440,14 +443,14 @@ __device__ __forceinline__ void row_attention(const RowStage& st, const RowGroup
   if (slot == 0 && on) *reinterpret_cast<MR_LDS v4f*>(part + (g.wave * L + c) * 4) = o;
   lds_store_barrier();
   const int n = min(wps, LP);
-  for (int t = g.wave * 64 + lane; t < g.nr * D; t += ROW_WAVES * 64) {
+  for (int t = g.wave * 64 + lane; t < g.nr * D; t += W * 64) {
     const int sq = t >= D ? 1 : 0, d = t - sq * D;   // at most 2 sequences
     const MR_LDS float* p = part + sq * wps * D + d;
-    float v[ROW_WAVES];
+    float v[W];
 #pragma unroll
-    for (int i = 0; i < ROW_WAVES; ++i) v[i] = p[min(i, n - 1) * D];
+    for (int i = 0; i < W; ++i) v[i] = p[min(i, n - 1) * D];
 #pragma unroll
-    for (int k = ROW_WAVES / 2; k > 0; k >>= 1)
+    for (int k = W / 2; k > 0; k >>= 1)
       if (k < n)
 #pragma unroll
         for (int i = 0; i < k; ++i) v[i] = __fadd_rn(v[i], v[i + k]);
@@ -456,7 +459,8 @@ __device__ __forceinline__ void row_attention(const RowStage& st, const RowGroup
 }
 
 // work_at: LDS offset of the attention's own part, behind the rows
-__global__ void __launch_bounds__(ROW_WAVES * 64) row_chain_kernel(uint64_t stages, int32_t n, int64_t rows, int32_t rpw,
+template <int W>
+__global__ void __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(4))) row_chain_kernel(uint64_t stages, int32_t n, int64_t rows, int32_t rpw,
                                                                   int32_t work_at) {
   extern __shared__ __attribute__((aligned(16))) char row_lds[];
   RowGroup g;
@@ -470,9 +474,9 @@ __global__ void __launch_bounds__(ROW_WAVES * 64) row_chain_kernel(uint64_t stag
   Ahead ahead;
   for (int i = 0; i < n; ++i) {
     const RowStage& st = *(const RowStage*)(first + i);
-    look_ahead(st, g, ahead);
+    look_ahead<W>(st, g, ahead);
     if (!(st.flags & ROW_NO_BARRIER)) lds_store_barrier();
-    if (g.wave == ROW_WAVES - 1 && i + 1 < n) {
+    if (g.wave == W - 1 && i + 1 < n) {
       const __attribute__((address_space(4))) int* next =
           reinterpret_cast<const __attribute__((address_space(4))) int*>(stages + (i + 1) * sizeof(RowStage));
       int any = 0;
@@ -484,14 +488,14 @@ __global__ void __launch_bounds__(ROW_WAVES * 64) row_chain_kernel(uint64_t stag
     // the kinds, it takes the registers past 128 and spills
     asm volatile("" : "+v"(g.lane));
     switch (st.kind) {
-      case ROW_LOAD: row_load(st, g); break;
-      case MR_ROW_QUANTIZE: row_quantize(st, g); break;
+      case ROW_LOAD: row_load<W>(st, g); break;
+      case MR_ROW_QUANTIZE: row_quantize<W>(st, g); break;
       case MR_ROW_LAYERNORM: row_layernorm(st, g, ahead); break;
-      case MR_ROW_QMATMUL: row_qmatmul(st, g, ahead); break;
+      case MR_ROW_QMATMUL: row_qmatmul<W>(st, g, ahead); break;
       default:
-        if (st.hd == 16) row_attention<16>(st, g, reinterpret_cast<MR_LDS float*>(g.lds + work_at));
-        else if (st.hd == 32) row_attention<32>(st, g, reinterpret_cast<MR_LDS float*>(g.lds + work_at));
-        else row_attention<64>(st, g, reinterpret_cast<MR_LDS float*>(g.lds + work_at));
+        if (st.hd == 16) row_attention<W, 16>(st, g, reinterpret_cast<MR_LDS float*>(g.lds + work_at));
+        else if (st.hd == 32) row_attention<W, 32>(st, g, reinterpret_cast<MR_LDS float*>(g.lds + work_at));
+        else row_attention<W, 64>(st, g, reinterpret_cast<MR_LDS float*>(g.lds + work_at));
     }
   }
 }
@@ -671,9 +675,16 @@ int mr_row_chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows, vo
   // one workgroup per CU while the rows allow it, with at most 2 sequences of an attention each
   // (its waves split the keys: at most 4 passes) or 16 rows without one
   const int64_t cus = device_cu_count();
-  const int most = !score_floats ? ROW_MAX_ROWS : wide <= 128 ? 2 : 1;
-  auto work = [&](int r) { return score_floats ? (((r * score_floats + 3) & ~int64_t(3)) + ROW_WAVES * 64 * 4) * 4 : 0; };
-  int rpw = 1;
+  int most = !score_floats ? ROW_MAX_ROWS : wide <= 128 ? 2 : 1;
+  int rpw = 1, waves = 16;
+  if (score_floats && rows > cus && wide <= 128) {
+    // two workgroups of 8 waves and one sequence share a CU, so that one's cache loads run under
+    // the other's short stages (512 sequences, D = 64: a two-layer step 59.9 -> 56.8 us, an
+    // attention half 20.1 -> 19.4); wider rows would take more than 4 passes
+    waves = 8;
+    most = 1;
+  }
+  auto work = [&](int r) { return score_floats ? (((r * score_floats + 3) & ~int64_t(3)) + waves * 64 * 4) * 4 : 0; };
   while (rpw < most && (rows + rpw - 1) / rpw > cus && work(2 * rpw) <= ROW_MAX_LDS) rpw *= 2;
 
   // which value each input is: rows an earlier stage wrote last, at the same stride (a column
@@ -777,16 +788,19 @@ int mr_row_chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows, vo
   plan[1] = static_cast<int32_t>(kept);
   plan[2] = static_cast<int32_t>(kept + work(rpw));
   plan[3] = static_cast<int32_t>(all.size());
+  plan[4] = waves;
   return MR_OK;
 }
 
 int mr_row_chain(const void* descriptors, int64_t rows, const int32_t* plan, void* stream) {
   MR_REQUIRE(descriptors && plan && rows >= 0, "mr_row_chain: bad argument");
   MR_REQUIRE(plan[0] >= 1 && plan[0] <= mr::ROW_MAX_ROWS && plan[1] >= 0 && plan[1] <= plan[2] &&
-             plan[2] <= mr::ROW_MAX_LDS && plan[3] > 0, "mr_row_chain: not a plan of mr_row_chain_prepare");
+             plan[2] <= mr::ROW_MAX_LDS && plan[3] > 0 &&
+             (plan[4] == 16 || (plan[4] == 8 && plan[0] <= 8)), "mr_row_chain: not a plan of mr_row_chain_prepare");
   if (rows == 0) return MR_OK;
   const unsigned grid = static_cast<unsigned>((rows + plan[0] - 1) / plan[0]);
-  hipLaunchKernelGGL(mr::row_chain_kernel, dim3(grid), dim3(mr::ROW_WAVES * 64), static_cast<unsigned>(plan[2]),
+  auto* kernel = plan[4] == 8 ? mr::row_chain_kernel<8> : mr::row_chain_kernel<16>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(plan[4] * 64), static_cast<unsigned>(plan[2]),
                      static_cast<hipStream_t>(stream), reinterpret_cast<uint64_t>(descriptors), plan[3], rows, plan[0],
                      plan[1]);
   MR_LAUNCH_CHECK("row_chain");

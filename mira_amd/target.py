@@ -110,9 +110,9 @@ F32IN_MAX_ROWS, F32IN_MAX_K = 8, 4096     # mr_qmatmul_f32in's decode shapes (k_
 LNIN_MAX_K = 1024                          # mr_qmatmul_lnin's rows (k_pad <= 1024)
 # Runs of row-local launches as one (_plan_row_chains): packed bytes of a q-op, and rows.  Four
 # K x K q-ops with two layernorms and residuals, us as launches / as a run (in a HIP graph):
-#   K = 64    1 row 17.9 / 14.3    512 rows 21.4 / 15.8    1024 rows 21.8 / 21.1
-#   K = 256   1 row 19.2 / 17.8    512 rows 27.4 / 20.6    1024 rows 28.0 / 27.1
-#   K = 384   1 row 19.5 / 26.2    512 rows 30.8 / 32.0    1024 rows 32.0 / 42.3
+#   K = 64    1 row 18.0 / 14.4    512 rows 21.5 / 15.8    1024 rows 21.8 / 21.4
+#   K = 256   1 row 19.3 / 17.8    512 rows 27.4 / 20.3    1024 rows 28.1 / 27.2
+#   K = 384   1 row 19.7 / 26.4    512 rows 30.8 / 31.9    1024 rows 31.9 / 42.6
 ROW_CHAIN_WEIGHTS, ROW_CHAIN_ROWS = 64 << 10, 512
 
 
@@ -617,7 +617,7 @@ class RocmExecutable:
                     s.flags |= L.ROW_ONLY_HERE_F32
         size = self.lib.mr_row_chain_bytes(n)
         host = np.zeros(size, np.uint8)
-        plan = (C.c_int32 * 4)()
+        plan = (C.c_int32 * 5)()
         rc = self.lib.mr_row_chain_prepare(arr, n, rows, host.ctypes.data, size, plan)
         if rc == L.EUNSUPPORTED:
             return None
