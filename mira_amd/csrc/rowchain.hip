@@ -23,8 +23,8 @@
 //    are loaded before the barrier in front of it.
 //
 // Measured, against the launches: the 16 of a two-layer D = 64 decode step over 272 keys for 512
-// sequences 140.4 -> 56.8 us; one sequence's greedy decode of it 69.0 -> 44.0 us a token, about 36
-// of them here (1.2-2 us a stage, 5.5 us an attention); one attention half (layernorm,
+// sequences 140.4 -> 56.8 us; one sequence's greedy decode of it 69.0 -> 44.0 us a token, 31 of
+// them here (1.2-2 us a stage, 5.5 us an attention); one attention half (layernorm,
 // projections, attention) of 512 sequences, 71 MB of cache, 23.7 -> 19.4; a quantize and a
 // 256 x 64 x 10 dense layer 10.8 -> 5.7.
 #include "mr_common.hpp"
@@ -32,6 +32,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <new>
 #include <vector>
 
 namespace mr {
@@ -518,19 +519,14 @@ struct RowValue {
   int64_t at;           // its place, or -1
 };
 
-}  // namespace mr
+static int64_t chain_bytes(int32_t n) { return n > 0 && n < (1 << 20) ? int64_t(2 * n + 8) * sizeof(RowStage) : -1; }
 
-extern "C" {
-
-int64_t mr_row_chain_bytes(int32_t n) { return n > 0 && n < (1 << 20) ? int64_t(2 * n + 8) * sizeof(mr::RowStage) : -1; }
-
-int mr_row_chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows, void* descriptors, int64_t bytes,
+static int chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows, void* descriptors, int64_t bytes,
                          int32_t* plan) {
-  using namespace mr;
   MR_REQUIRE(stages && descriptors && plan && n > 0 && n < (1 << 20), "mr_row_chain_prepare: NULL argument or no stage");
   MR_REQUIRE(rows >= 0 && rows < (int64_t(1) << 31), "mr_row_chain_prepare: bad row count %lld", (long long)rows);
-  MR_REQUIRE(bytes >= mr_row_chain_bytes(n), "mr_row_chain_prepare: descriptors need %lld bytes",
-             (long long)mr_row_chain_bytes(n));
+  MR_REQUIRE(bytes >= chain_bytes(n), "mr_row_chain_prepare: descriptors need %lld bytes",
+             (long long)chain_bytes(n));
   std::vector<RowStage> out(n);
   std::memset(out.data(), 0, n * sizeof(RowStage));
   int64_t score_floats = 0, wide = 0;     // per row, the largest attention's scores; its columns
@@ -790,6 +786,22 @@ int mr_row_chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows, vo
   plan[3] = static_cast<int32_t>(all.size());
   plan[4] = waves;
   return MR_OK;
+}
+
+}  // namespace mr
+
+extern "C" {
+
+int64_t mr_row_chain_bytes(int32_t n) { return mr::chain_bytes(n); }
+
+int mr_row_chain_prepare(const mr_row_stage* stages, int32_t n, int64_t rows, void* descriptors, int64_t bytes,
+                         int32_t* plan) {
+  try {
+    return mr::chain_prepare(stages, n, rows, descriptors, bytes, plan);
+  } catch (const std::bad_alloc&) {
+    mr::set_error("mr_row_chain_prepare: out of host memory");
+    return MR_EUNSUPPORTED;
+  }
 }
 
 int mr_row_chain(const void* descriptors, int64_t rows, const int32_t* plan, void* stream) {
