@@ -417,8 +417,8 @@ def bench_gpt(args) -> int:
         "exact_mode_host_loop_us_per_step": round(1e6 * host_s / host_steps, 1),
         "exact_mode_host_loop_steps": host_steps,
         "exact_mode_segments": host_runner.devices,
-        "launches_per_step": len(exe.launches) + 2,          # the step, and the loop's embed and commit kernels
-        "step_launches": len(exe.launches),
+        "launches_per_step": len(exe.program) + 2,          # the step, and the loop's embed and commit kernels
+        "step_launches": len(exe.program),
         "device_constant_bytes": exe.const_bytes,
         "dtype": "int8", "data": "synthetic",
         "timed": "HIP events around every decode step of the prompt and the generated tokens, the step "

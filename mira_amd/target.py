@@ -2392,7 +2392,7 @@ class RocmExecutable:
 
     def report(self) -> str:
         ks = ", ".join(f"{k} x{n}" for k, n in sorted(self.kernel_counts.items()))
-        return (f"rocm (MI355X gfx950): {len(self.g.compute_ops())} ops -> {len(self.launches)} kernel launches "
+        return (f"rocm (MI355X gfx950): {len(self.g.compute_ops())} ops -> {len(self.program)} kernel launches "
                 f"[{ks}]; {self.const_bytes / 2**20:.2f} MiB of packed constants on device")
 
 
